@@ -183,7 +183,8 @@ void sh_conv_destroy(sh_conv *c);
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc. No
  * reference counterpart (ConvEval allocates its IOSurfaces per kernel). x [s, in_dim] and out
  * [s, out_dim] are device pointers the caller owns; the work is enqueued on `stream` (a
- * hipStream_t; NULL = the null stream) and the call returns without waiting. The input's
+ * hipStream_t; NULL = the null stream) and the call returns without waiting. out may equal x or
+ * overlap it: every row of x is read before it is overwritten. The input's
  * operand planes and the product's K-range partials live in a static 16 MiB device array
  * per GPU (resolved at sh_init); a call whose planes (4*s*in_dim bytes) need more fails with a
  * message saying how much (partials that no longer fit beside the planes are not used: the

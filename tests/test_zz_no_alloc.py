@@ -74,3 +74,32 @@ def test_conv_eval_noalloc_matches_conv_eval(gpu, out_dim, in_dim):
         hip.free(dx)
         hip.free(dy)
         conv.close()
+
+
+@pytest.mark.parametrize("s,out_dim,in_dim", [
+    (1, 768, 768), (16, 768, 768), (16, 2048, 4096), (32, 1024, 1024), (128, 768, 768),   # one launch for all
+    (300, 768, 768), (957, 1024, 1024), (40, 1088, 2016)])                                 # operand planes, then the product
+def test_conv_eval_noalloc_over_its_own_input(gpu, s, out_dim, in_dim):
+    """out == x, and out begun before and inside x (by whole rows and by a few floats): every row of
+    x is read before it is overwritten, so the results are sh_conv_eval's bits."""
+    lib = sh.load()
+    hip = Hip()
+    rng = np.random.default_rng(191 + s)
+    conv = sh.Conv((rng.standard_normal((out_dim, in_dim)) * 0.05).astype(np.float32))
+    x = rng.standard_normal((s, in_dim)).astype(np.float32)
+    want = conv.eval(x)
+    pad = max(in_dim, out_dim)
+    n = s * pad + 2 * pad
+    buf = hip.malloc(4 * n)
+    try:
+        for shift in (0, 3, -5, pad, -pad, (s // 2) * in_dim):
+            at_x, at_out = 4 * pad, 4 * (pad + min(shift, n - pad - s * out_dim))
+            hip.h2d(C.c_void_p(buf.value + at_x), x)
+            assert lib.sh_conv_eval_noalloc(conv.h, buf.value + at_x, s, buf.value + at_out, None) == 0, sh.last_error()
+            hip.sync()
+            got = np.empty((s, out_dim), np.float32)
+            hip.d2h(got, C.c_void_p(buf.value + at_out))
+            np.testing.assert_array_equal(got, want, err_msg=f"out {shift} floats after x")
+    finally:
+        hip.free(buf)
+        conv.close()
