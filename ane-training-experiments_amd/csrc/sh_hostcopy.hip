@@ -2,17 +2,12 @@
 #include "sh_hostcopy.hpp"
 
 #include <stdint.h>
-#include <string.h>
-#include <sys/mman.h>
-#include <unistd.h>
 
 #include <algorithm>
-#include <atomic>
-#include <condition_variable>
 #include <exception>
-#include <mutex>
 #include <thread>
-#include <vector>
+
+#include "sh_copypool.hpp"
 
 namespace sh {
 namespace {
@@ -21,20 +16,7 @@ constexpr size_t kMin = 512u << 10;     // smaller copies: the runtime's own pat
 constexpr int kOutBlocks = 128, kOutThreads = 256;
 constexpr size_t kSlot = 2u << 20;
 constexpr int kSlots = 4;
-constexpr int kMaxThreads = 6;
-constexpr int kSpins = 20000;           // about 0.2 ms of pauses before a worker sleeps
-
-#ifndef MADV_POPULATE_WRITE
-#define MADV_POPULATE_WRITE 23          // Linux 5.14; older kernels answer EINVAL
-#endif
-
-// One job at a time, split evenly over the workers: dst[0, n) copied from src, or, without a
-// src, its pages faulted in.
-struct Job {
-    uint8_t *dst = nullptr;
-    const uint8_t *src = nullptr;
-    size_t n = 0;
-};
+constexpr int kMaxHelpers = 5;
 
 // n16 16-byte words to pinned host memory, then `tail` bytes: a launch starts sooner than a
 // transfer of the copy engines, whose first use by a process costs about 1.5 ms.
@@ -44,78 +26,26 @@ __global__ __launch_bounds__(kOutThreads) void k_copy_out(const uint4 *src, uint
     if (i0 < (size_t)tail) ((uint8_t *)(dst + n16))[i0] = ((const uint8_t *)(src + n16))[i0];
 }
 
-void run_part(const Job &j, int part, int parts) {
-    const size_t a = j.n * part / parts & ~(size_t)63, b = part + 1 == parts ? j.n : j.n * (part + 1) / parts & ~(size_t)63;
-    if (j.src) {
-        memcpy(j.dst + a, j.src + a, b - a);
-    } else if (b > a) {
-        const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE);
-        const uintptr_t lo = ((uintptr_t)j.dst + a) & ~(page - 1), hi = ((uintptr_t)j.dst + b + page - 1) & ~(page - 1);
-        (void)madvise((void *)lo, hi - lo, MADV_POPULATE_WRITE);   // a failure leaves the faults to the copy
-    }
-}
-
 }  // namespace
 
 struct HostCopier::State {
     uint8_t *ring = nullptr;
     hipEvent_t ev[kSlots] = {};
     bool recorded[kSlots] = {};
-    std::vector<std::thread> threads;
-    std::mutex mu;
-    std::condition_variable cv;
-    Job job;                           // written before `posted` moves, read after
-    std::atomic<uint64_t> posted{0};   // jobs handed out
-    std::atomic<uint64_t> parts{0};    // parts finished, over all jobs
-    std::atomic<int> sleeping{0};
-    std::atomic<bool> stop{false};
-
-    void work(int me, int of) {
-        uint64_t seen = 0;
-        for (;;) {
-            for (int i = 0; i < kSpins && posted.load() == seen && !stop.load(); i++) __builtin_ia32_pause();
-            if (posted.load() == seen && !stop.load()) {
-                std::unique_lock<std::mutex> lk(mu);
-                sleeping++;
-                cv.wait(lk, [&] { return posted.load() != seen || stop.load(); });
-                sleeping--;
-            }
-            if (stop.load()) return;
-            seen++;                    // the next job is posted only after this one's parts are done
-            run_part(job, me, of);
-            parts++;
-        }
-    }
-    void wait() const {
-        const uint64_t all = posted.load() * threads.size();
-        while (parts.load() != all) __builtin_ia32_pause();
-    }
-    void post(void *dst, const void *src, size_t n) {
-        wait();
-        job = Job{(uint8_t *)dst, (const uint8_t *)src, n};
-        posted++;
-        if (sleeping.load() > 0) {
-            std::lock_guard<std::mutex> lk(mu);
-            cv.notify_all();
-        }
-    }
+    CopyPool pool{std::max(1, std::min(kMaxHelpers, (int)std::thread::hardware_concurrency() / 2 - 1))};
 };
 
 bool HostCopier::ready() {
     if (st_ || refused_) return st_ != nullptr;
-    State *s = new State;
-    bool ok = hipHostMalloc((void **)&s->ring, kSlots * kSlot, hipHostMallocDefault) == hipSuccess;
-    for (int i = 0; ok && i < kSlots; i++) ok = hipEventCreateWithFlags(&s->ev[i], hipEventDisableTiming) == hipSuccess;
-    const int hw = (int)std::thread::hardware_concurrency();
-    const int want = std::max(1, std::min(kMaxThreads, hw / 2 - 1));
     try {
-        s->threads.reserve(want);
-        // each worker's share is fixed by the final count, so none runs before all exist
-        for (int i = 0; ok && i < want; i++) s->threads.emplace_back([s, i, want] { s->work(i, want); });
+        st_ = new State;
     } catch (const std::exception &) {
-        ok = false;
+        refused_ = true;
+        return false;
     }
-    st_ = s;
+    bool ok = hipHostMalloc((void **)&st_->ring, kSlots * kSlot, hipHostMallocDefault) == hipSuccess;
+    for (int i = 0; ok && i < kSlots; i++)
+        ok = hipEventCreateWithFlags(&st_->ev[i], hipEventDisableTiming) == hipSuccess;
     if (ok) return true;
     (void)hipGetLastError();
     release();
@@ -125,14 +55,7 @@ bool HostCopier::ready() {
 
 void HostCopier::release() {
     if (!st_) return;
-    if (st_->threads.size()) {
-        st_->stop = true;
-        {
-            std::lock_guard<std::mutex> lk(st_->mu);
-            st_->cv.notify_all();
-        }
-        for (auto &t : st_->threads) t.join();
-    }
+    st_->pool.finish();
     for (hipEvent_t e : st_->ev)
         if (e) (void)hipEventDestroy(e);
     if (st_->ring) (void)hipHostFree(st_->ring);
@@ -141,10 +64,10 @@ void HostCopier::release() {
 }
 
 HostCopier::Prefault::Prefault(HostCopier &c, void *dst, size_t n) : c_(c) {
-    if (n >= kMin && c.ready()) c.st_->post(dst, nullptr, n);
+    if (n >= kMin && c.ready()) c.st_->pool.start(dst, nullptr, n);
 }
 HostCopier::Prefault::~Prefault() {
-    if (c_.st_) c_.st_->wait();
+    if (c_.st_) c_.st_->pool.finish();
 }
 
 // Eight chunks or more, so that the DMA of one runs beside the host copies of others.
@@ -176,11 +99,11 @@ hipError_t HostCopier::to_host(void *dst, const void *src, size_t n, hipStream_t
         e = hipEventSynchronize(st_->ev[i % kSlots]);
         if (e != hipSuccess) break;
         const size_t o = i * chunk;
-        st_->post((uint8_t *)dst + o, st_->ring + (i % kSlots) * kSlot, std::min(chunk, n - o));
-        // posting chunk i waited for chunk i - 1's copy, whose slot is the next one to fill
+        st_->pool.start((uint8_t *)dst + o, st_->ring + (i % kSlots) * kSlot, std::min(chunk, n - o));
+        // starting chunk i finished chunk i - 1's copy, whose slot is the next one to fill
         if (i + kSlots - 1 < nc) fetch(i + kSlots - 1);
     }
-    st_->wait();
+    st_->pool.finish();
     if (e != hipSuccess) (void)hipStreamSynchronize(s);   // nothing may still write the ring
     return e;
 }
@@ -192,14 +115,14 @@ hipError_t HostCopier::to_device(void *dst, const void *src, size_t n, hipStream
     const auto stage = [&](int i) -> hipError_t {   // once the slot's last transfer, of any call, is done
         const int k = i % kSlots;
         const hipError_t e = st_->recorded[k] ? hipEventSynchronize(st_->ev[k]) : hipSuccess;
-        if (e == hipSuccess) st_->post(st_->ring + k * kSlot, (const uint8_t *)src + i * chunk, std::min(chunk, n - i * chunk));
+        if (e == hipSuccess) st_->pool.start(st_->ring + k * kSlot, (const uint8_t *)src + i * chunk, std::min(chunk, n - i * chunk));
         return e;
     };
     hipError_t e = stage(0);
     for (int i = 0; e == hipSuccess && i < nc; i++) {
-        // staging chunk i + 1 waits for chunk i's host copy and then runs beside its transfer
+        // staging chunk i + 1 finishes chunk i's host copy and then runs beside its transfer
         if (i + 1 < nc) e = stage(i + 1);
-        else st_->wait();
+        else st_->pool.finish();
         if (e != hipSuccess) break;
         const int k = i % kSlots;
         const size_t o = i * chunk;
@@ -207,7 +130,7 @@ hipError_t HostCopier::to_device(void *dst, const void *src, size_t n, hipStream
         if (e == hipSuccess) e = hipEventRecord(st_->ev[k], s);
         st_->recorded[k] = e == hipSuccess;
     }
-    st_->wait();
+    st_->pool.finish();
     if (e != hipSuccess) (void)hipStreamSynchronize(s);   // nothing may still read the ring
     return e;
 }
