@@ -293,7 +293,7 @@ bool seam_begin(sh_model *m, const char *what, const float *x_cf, int32_t seq, v
     const size_t xb = sizeof(float) * (size_t)m->cfg.dim * seq;
     return hip_ok(hipMemcpyAsync(m->pf_rowpos, rows.data(), 4 * (size_t)seq, hipMemcpyHostToDevice, m->stream), "seam rows") &&
            hip_ok(hipMemcpyAsync(m->pf_rowseq, rows.data() + seq, 4 * (size_t)seq, hipMemcpyHostToDevice, m->stream), "seam rows") &&
-           hip_ok(m->copier.to_device(m->pf_cf, x_cf, xb, m->stream), "seam input") &&
+           hip_ok(hipMemcpyAsync(m->pf_cf, x_cf, xb, hipMemcpyHostToDevice, m->stream), "seam input") &&
            hip_ok(hipEventRecord(m->ev0, m->stream), "event");
 }
 

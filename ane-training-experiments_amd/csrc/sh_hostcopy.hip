@@ -12,18 +12,21 @@
 namespace sh {
 namespace {
 
-constexpr size_t kMin = 512u << 10;     // smaller copies: the runtime's own path is as fast
+// Smaller copies take the runtime's own path. Into warm pages, called every 2 ms (the helpers asleep):
+// 1 MiB 63 us by the runtime and 80 through the ring, 2 MiB 122 and 129, 3 MiB 185 and 131, 32 MiB
+// 1878 and 707; into fresh pages 2 MiB 480 and 362. (The other way the runtime is as fast up to 16
+// MiB: 2 MiB in 80 us against 201 through the ring.)
+constexpr size_t kMin = 2u << 20;
 constexpr int kOutBlocks = 128, kOutThreads = 256;
 constexpr size_t kSlot = 2u << 20;
 constexpr int kSlots = 4;
 constexpr int kMaxHelpers = 5;
 
-// n16 16-byte words to pinned host memory, then `tail` bytes: a launch starts sooner than a
-// transfer of the copy engines, whose first use by a process costs about 1.5 ms.
-__global__ __launch_bounds__(kOutThreads) void k_copy_out(const uint4 *src, uint4 *dst, size_t n16, int tail) {
-    const size_t i0 = (size_t)blockIdx.x * kOutThreads + threadIdx.x;
-    for (size_t i = i0; i < n16; i += (size_t)kOutBlocks * kOutThreads) dst[i] = src[i];
-    if (i0 < (size_t)tail) ((uint8_t *)(dst + n16))[i0] = ((const uint8_t *)(src + n16))[i0];
+// n16 16-byte words to pinned host memory: a launch starts sooner than a transfer of the copy
+// engines, whose first use by a process costs about 1.5 ms.
+__global__ __launch_bounds__(kOutThreads) void k_copy_out(const uint4 *src, uint4 *dst, size_t n16) {
+    for (size_t i = (size_t)blockIdx.x * kOutThreads + threadIdx.x; i < n16; i += (size_t)kOutBlocks * kOutThreads)
+        dst[i] = src[i];
 }
 
 }  // namespace
@@ -31,7 +34,6 @@ __global__ __launch_bounds__(kOutThreads) void k_copy_out(const uint4 *src, uint
 struct HostCopier::State {
     uint8_t *ring = nullptr;
     hipEvent_t ev[kSlots] = {};
-    bool recorded[kSlots] = {};
     CopyPool pool{std::max(1, std::min(kMaxHelpers, (int)std::thread::hardware_concurrency() / 2 - 1))};
 };
 
@@ -74,24 +76,20 @@ HostCopier::Prefault::~Prefault() {
 static size_t chunk_of(size_t n) { return std::min(kSlot, std::max<size_t>(256u << 10, (n / 8 + 65535) & ~(size_t)65535)); }
 
 hipError_t HostCopier::to_host(void *dst, const void *src, size_t n, hipStream_t s) {
-    if (n < kMin || !ready()) {
+    if (n < kMin || n % 16 || (uintptr_t)src % 16 || !ready()) {
         const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, s);
         return e != hipSuccess ? e : hipStreamSynchronize(s);
     }
+    uint8_t *ring = st_->ring;
+    CopyPool &pool = st_->pool;
     const size_t chunk = chunk_of(n);
     const int nc = (int)((n + chunk - 1) / chunk);
     hipError_t e = hipSuccess;
     const auto fetch = [&](int i) {
         const size_t o = i * chunk, m = std::min(chunk, n - o);
-        uint8_t *slot = st_->ring + (i % kSlots) * kSlot;
-        const uint8_t *from = (const uint8_t *)src + o;
-        if ((uintptr_t)src % 16) {
-            e = hipMemcpyAsync(slot, from, m, hipMemcpyDeviceToHost, s);
-        } else {
-            hipLaunchKernelGGL(k_copy_out, dim3(kOutBlocks), dim3(kOutThreads), 0, s, (const uint4 *)from,
-                               (uint4 *)slot, m / 16, (int)(m % 16));
-            e = hipGetLastError();
-        }
+        hipLaunchKernelGGL(k_copy_out, dim3(kOutBlocks), dim3(kOutThreads), 0, s, (const uint4 *)((const uint8_t *)src + o),
+                           (uint4 *)(ring + (i % kSlots) * kSlot), m / 16);
+        e = hipGetLastError();
         if (e == hipSuccess) e = hipEventRecord(st_->ev[i % kSlots], s);
     };
     for (int i = 0; e == hipSuccess && i < std::min(nc, kSlots - 1); i++) fetch(i);
@@ -99,39 +97,12 @@ hipError_t HostCopier::to_host(void *dst, const void *src, size_t n, hipStream_t
         e = hipEventSynchronize(st_->ev[i % kSlots]);
         if (e != hipSuccess) break;
         const size_t o = i * chunk;
-        st_->pool.start((uint8_t *)dst + o, st_->ring + (i % kSlots) * kSlot, std::min(chunk, n - o));
+        pool.start((uint8_t *)dst + o, ring + (i % kSlots) * kSlot, std::min(chunk, n - o));
         // starting chunk i finished chunk i - 1's copy, whose slot is the next one to fill
         if (i + kSlots - 1 < nc) fetch(i + kSlots - 1);
     }
-    st_->pool.finish();
+    pool.finish();
     if (e != hipSuccess) (void)hipStreamSynchronize(s);   // nothing may still write the ring
-    return e;
-}
-
-hipError_t HostCopier::to_device(void *dst, const void *src, size_t n, hipStream_t s) {
-    if (n < kMin || !ready()) return hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, s);
-    const size_t chunk = chunk_of(n);
-    const int nc = (int)((n + chunk - 1) / chunk);
-    const auto stage = [&](int i) -> hipError_t {   // once the slot's last transfer, of any call, is done
-        const int k = i % kSlots;
-        const hipError_t e = st_->recorded[k] ? hipEventSynchronize(st_->ev[k]) : hipSuccess;
-        if (e == hipSuccess) st_->pool.start(st_->ring + k * kSlot, (const uint8_t *)src + i * chunk, std::min(chunk, n - i * chunk));
-        return e;
-    };
-    hipError_t e = stage(0);
-    for (int i = 0; e == hipSuccess && i < nc; i++) {
-        // staging chunk i + 1 finishes chunk i's host copy and then runs beside its transfer
-        if (i + 1 < nc) e = stage(i + 1);
-        else st_->pool.finish();
-        if (e != hipSuccess) break;
-        const int k = i % kSlots;
-        const size_t o = i * chunk;
-        e = hipMemcpyAsync((uint8_t *)dst + o, st_->ring + k * kSlot, std::min(chunk, n - o), hipMemcpyHostToDevice, s);
-        if (e == hipSuccess) e = hipEventRecord(st_->ev[k], s);
-        st_->recorded[k] = e == hipSuccess;
-    }
-    st_->pool.finish();
-    if (e != hipSuccess) (void)hipStreamSynchronize(s);   // nothing may still read the ring
     return e;
 }
 

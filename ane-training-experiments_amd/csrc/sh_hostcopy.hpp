@@ -1,11 +1,10 @@
-// sh_hostcopy.hpp — large copies between a caller's ordinary (pageable) memory and the device.
+// sh_hostcopy.hpp — large results copied into a caller's ordinary (pageable) memory.
 //
-// The entry points take and return host arrays, so a full-sequence forward's logits (32.8 MB for
-// Stories110M at 256 positions) cross PCIe into pages the caller has often just mapped. The
-// runtime's own copy of pageable memory pins or stages it on one thread: 17 GB/s into warm pages,
-// 9 into fresh ones (faulting 32 MB alone takes 1.3 ms), against 56 GB/s of PCIe into pinned
-// memory. Here the transfer runs through a small pinned ring, a few threads move the other half
-// of the way (one moves 16 GB/s), and the result's pages are faulted in while the GPU still
+// The entry points return host arrays, so a full-sequence forward's logits (32.8 MB for Stories110M
+// at 256 positions) cross PCIe into pages the caller has often just mapped. The runtime's own copy
+// moves 17 GB/s into warm pages and, faulting them on its one thread, 4 to 9 into fresh ones, against
+// 56 GB/s of PCIe into pinned memory. Here the transfer runs through a small pinned ring, a few
+// threads move the other half of the way, and the result's pages are faulted in while the GPU still
 // computes it.
 #pragma once
 
@@ -38,8 +37,6 @@ class HostCopier {
     };
     // Copies n device bytes to dst after the stream's earlier work; dst is complete on return.
     hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s);
-    // Enqueues the copy of n host bytes to the device; src has been read on return.
-    hipError_t to_device(void *dst, const void *src, size_t n, hipStream_t s);
 
   private:
     struct State;

@@ -87,7 +87,7 @@ struct sh_model {
     sh::DecodeState *state;
     int32_t *step_host;    // pinned: a decode step's results ({argmax, error word, -, -}, logits [V])
 
-    sh::HostCopier copier;   // large host arrays in and out, on `stream`
+    sh::HostCopier copier;   // large results to host arrays, on `stream`
 
     hipGraphExec_t step_exec;
     bool step_ready;

@@ -1,7 +1,6 @@
 """Large results copied to host arrays (HostCopier) bit for bit: sizes around its threshold
-(512 KiB), of an uneven last chunk and beyond its pinned ring (8 MiB), at unaligned host
-addresses, through a trainer's embedding [V, D] read back. (Its other direction carries the
-layer seam's inputs, which test_gpu_gemm.py compares with the oracle at 0.6 to 3.4 MB.)"""
+(2 MiB), of an uneven last chunk and beyond its pinned ring (8 MiB), at unaligned host
+addresses, through a trainer's embedding [V, D] read back."""
 import ctypes as C
 
 import numpy as np
@@ -13,7 +12,7 @@ from helpers import tiny_config
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("vocab", [2044, 2048, 2052, 8188, 32772, 65532])   # rows of 256 bytes
+@pytest.mark.parametrize("vocab", [2048, 8188, 8192, 8196, 9004, 32772, 65532])   # rows of 256 bytes
 def test_read_round_trip(gpu, vocab):
     cfg = tiny_config(dim=64, hidden=128, n_layers=1, n_heads=4, n_kv_heads=4, head_dim=16, vocab=vocab, max_seq=32)
     tr = sh.Trainer(cfg, seq=16)
