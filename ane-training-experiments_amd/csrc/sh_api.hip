@@ -693,7 +693,6 @@ int sh_model_upload_layer(sh_model *m, int32_t layer, const float *wq, const flo
     (void)hipSetDevice(m->device);
     const int D = c.dim, F = c.hidden;
     const size_t biggest = std::max({(size_t)m->qdim * D, (size_t)F * D});
-    if (biggest >= (1u << 20)) m->copier.prepare();   // a model whose activations and logits are large
     float *staging = nullptr;
     if (!hip_ok(hipMalloc(&staging, biggest * 4), "hipMalloc staging")) return -1;
     LayerDev &L = m->layers[layer];

@@ -14,17 +14,16 @@
 namespace sh {
 
 // Owned by one model or trainer and used, like it, by one thread at a time, always with the
-// owner's stream. The pinned ring (8 MiB) and the threads come with prepare() or the first
-// large copy and go with the object; without them (allocation refused) the runtime's copy is
-// used.
+// owner's stream. The copiers of a process share one pinned ring (8 MiB) and its threads, one copy
+// at a time: they come once the process has copied 32 MiB of large results without them, and go
+// with the last object that used them. Without them (not set up yet, another thread's copy has
+// them, allocation refused) the runtime's copy is used.
 class HostCopier {
   public:
     HostCopier() = default;
     HostCopier(const HostCopier &) = delete;
     HostCopier &operator=(const HostCopier &) = delete;
     ~HostCopier() { release(); }
-    // Sets the ring and the threads up now (about 1 ms), outside any timed call.
-    void prepare() { (void)ready(); }
     // Faults in dst[0, n) beside whatever the caller does while the object lives; the contents
     // do not change.
     class Prefault {
@@ -34,13 +33,15 @@ class HostCopier {
 
       private:
         HostCopier &c_;
+        const bool on_;
     };
     // Copies n device bytes to dst after the stream's earlier work; dst is complete on return.
     hipError_t to_host(void *dst, const void *src, size_t n, hipStream_t s);
 
   private:
     struct State;
-    bool ready();
+    bool hold(size_t n);   // true: the ring is this copier's until let_go()
+    void let_go();
     void release();
     State *st_ = nullptr;
     bool refused_ = false;
