@@ -1,0 +1,19 @@
+"""Rules of csrc/sh_gemm_plan.hpp that keep a product's precision, over the sizes models can have."""
+import itertools
+
+from plan import plans
+
+# what dim, n_heads*head_dim and hidden can be
+WIDTHS = (64, 128, 192, 256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096)
+ROWS = (1, 4, 31, 64, 130, 255, 256, 257, 500, 1023, 1024, 1500, 4096)
+COLS = sorted({*WIDTHS, *(2 * w for w in WIDTHS), 320, 2304, 16320, 16384, 32000, 50304})
+
+
+def test_one_plane_where_it_has_always_been():
+    """Long inputs and wide classifiers took one plane with K a multiple of 128 (each of their K
+    ranges was one then), others from three K steps of 64 on; everything else kept the pair."""
+    products = list(itertools.product(ROWS, COLS, WIDTHS, (1,)))
+    for (m, n, k, _), p in zip(products, plans(products)):
+        large = (m >= 1024 or (m >= 256 and n >= 16384)) and n % 128 == 0
+        want = k % 128 == 0 if large else k // 64 >= 3
+        assert p.one_plane_ok == want, (m, n, k)

@@ -104,3 +104,30 @@ def test_eval_logits_on_ring_tiles(gpu, dtype, seq, vocab):
     err = float(np.max(np.abs(got - want)))
     print(f"S={seq} V={vocab}: max-abs {err:.2e}")
     assert err <= 2e-2
+
+
+@pytest.mark.parametrize("dim,hidden,vocab,seq", [
+    (64, 64, 512, 47), (128, 128, 512, 47), (64, 128, 512, 1100),   # every product
+    (192, 64, 16384, 256), (64, 64, 16384, 300),                    # a large classifier
+])
+def test_eval_logits_of_short_k_keep_the_pair(gpu, dim, hidden, vocab, seq):
+    """Products over 64, 128 or (large ones) 192 columns take the activations as a hi/lo pair also in
+    EvalLogits' fp16 form: relative error (2-norm) below 1e-5, where one fp16 plane makes 1e-4 or more (an
+    11-bit significand: 2^-12 / sqrt(3) of each activation). Wo is zero, so the attention, which takes one plane,
+    has no part in it, and so is W2 where W1|W3 take one plane."""
+    cfg = tiny_config(dim=dim, hidden=hidden, n_layers=2, n_heads=dim // 32, n_kv_heads=dim // 32, head_dim=32, vocab=vocab,
+                      max_seq=seq)
+    w = sh.synth_weights(cfg, seed=91 + dim, std=0.08)
+    for lw in w.layers:
+        lw["wo"] = np.zeros_like(lw["wo"])
+        if dim == 192:
+            lw["w2"] = np.zeros_like(lw["w2"])
+    m = sh.Model(cfg, sh.SH_DTYPE_F16)
+    m.upload(w)
+    toks = sh.synth_tokens(seq, 92, cfg.vocab).astype(np.uint16)
+    got = m.eval_logits(toks)
+    m.close()
+    want = oracle.eval_logits_cf(oracle.config_from(cfg), w.rounded(sh.SH_DTYPE_F16), toks, threads=THREADS)
+    err = float(np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want.astype(np.float64)))
+    print(f"rel {err:.2e}")
+    assert err <= 1e-5
