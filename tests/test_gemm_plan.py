@@ -17,3 +17,14 @@ def test_one_plane_where_it_has_always_been():
         large = (m >= 1024 or (m >= 256 and n >= 16384)) and n % 128 == 0
         want = k % 128 == 0 if large else k // 64 >= 3
         assert p.one_plane_ok == want, (m, n, k)
+
+
+def test_pairs_keep_sums_of_their_own():
+    """A pair's lo products have a sum apart from the hi products' (k_gemm_ring's SEP) in all tiles but
+    the widest, which only large products take."""
+    products = [(m, n, k, 0) for m, n, k in itertools.product((*ROWS, 193, 700, 900), (*COLS, 6144, 2112), (*WIDTHS, 416, 1568))]
+    for (m, n, k, _), p in zip(products, plans(products)):
+        large = (m >= 1024 or (m >= 256 and n >= 16384)) and n % 128 == 0
+        assert large or p.kind != "ring128x256", (m, n, k)
+    # sizes that took them: two rounds of the next smaller tile
+    assert {p.kind for p in plans([(193, 32000, 768, 0), (700, 6144, 2048, 0), (1000, 6144, 2048, 0)])} == {"ring128x128", "ring64x128"}
