@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -297,11 +298,20 @@ bool seam_begin(sh_model *m, const char *what, const float *x_cf, int32_t seq, v
            hip_ok(hipEventRecord(m->ev0, m->stream), "event");
 }
 
-// Copies `bytes` of device results to the host, waits, and records the device time.
-bool seam_end(sh_model *m, const void *dev, void *host, size_t bytes, int seq) {
+// Records the end of the device time, then copies the seam's results to the host and waits.
+struct SeamOut {
+    float *host;         // null: not asked for
+    const float *dev;
+    size_t n;
+};
+bool seam_end(sh_model *m, int seq, std::initializer_list<SeamOut> outs) {
     if (!hip_ok(hipEventRecord(m->ev1, m->stream), "event")) return false;
-    const HostCopier::Prefault pages(m->copier, host, bytes);   // while the seam's kernels run
-    if (!hip_ok(m->copier.to_host(host, dev, bytes, m->stream), "seam output")) return false;
+    for (const SeamOut &o : outs) {
+        if (!o.host) continue;
+        const size_t bytes = sizeof(float) * o.n;
+        const HostCopier::Prefault pages(m->copier, o.host, bytes);   // while the seam's kernels run
+        if (!hip_ok(m->copier.to_host(o.host, o.dev, bytes, m->stream), "seam output")) return false;
+    }
     float ms = 0;
     (void)hipEventElapsedTime(&ms, m->ev0, m->ev1);
     m->last = sh_timing{};
@@ -1612,7 +1622,7 @@ int sh_layer_forward_cf(sh_model *m, int32_t layer, const float *x_cf, int32_t s
     }
     if (!seam_begin(m, "sh_layer_forward_cf", x_cf, seq, out_cf, false, false)) return -1;
     if (!hip_ok(enqueue_layer_cf(m, layer, seq), "layer forward")) return -1;
-    return seam_end(m, m->pf_cf, out_cf, sizeof(float) * (size_t)m->cfg.dim * seq, seq) ? 0 : -1;
+    return seam_end(m, seq, {{out_cf, m->pf_cf, (size_t)m->cfg.dim * seq}}) ? 0 : -1;
 }
 
 int sh_layer_forward_cf_taps(sh_model *m, int32_t layer, const float *x_cf, int32_t seq,
@@ -1640,23 +1650,19 @@ int sh_layer_forward_cf_taps(sh_model *m, int32_t layer, const float *x_cf, int3
         !hip_ok(enqueue_layer_taps_cf(m, layer, seq, sdpa_cf ? d_sdpa : nullptr, ffn_cf ? d_ffn : nullptr,
                                       d_h13), "layer taps"))
         return -1;
-    if (sdpa_cf && !hip_ok(m->copier.to_host(sdpa_cf, d_sdpa, sizeof(float) * n_sdpa, m->stream), "sdpa taps"))
-        return -1;
-    if (ffn_cf && !hip_ok(m->copier.to_host(ffn_cf, d_ffn, sizeof(float) * n_ffn, m->stream), "ffn taps"))
-        return -1;
-    return seam_end(m, m->pf_cf, out_cf, sizeof(float) * (size_t)c.dim * seq, seq) ? 0 : -1;
+    return seam_end(m, seq, {{sdpa_cf, d_sdpa, n_sdpa}, {ffn_cf, d_ffn, n_ffn}, {out_cf, m->pf_cf, c.dim * S}}) ? 0 : -1;
 }
 
 int sh_rms_final_cf(sh_model *m, const float *x_cf, int32_t seq, float *out_cf) {
     if (!seam_begin(m, "sh_rms_final_cf", x_cf, seq, out_cf, false, true)) return -1;
     if (!hip_ok(enqueue_rms_final_cf(m, seq), "final rmsnorm")) return -1;
-    return seam_end(m, m->pf_cf, out_cf, sizeof(float) * (size_t)m->cfg.dim * seq, seq) ? 0 : -1;
+    return seam_end(m, seq, {{out_cf, m->pf_cf, (size_t)m->cfg.dim * seq}}) ? 0 : -1;
 }
 
 int sh_classifier_cf(sh_model *m, const float *xnorm_cf, int32_t seq, float *logits_cf) {
     if (!seam_begin(m, "sh_classifier_cf", xnorm_cf, seq, logits_cf, true, true)) return -1;
     if (!hip_ok(enqueue_classifier_cf(m, seq), "classifier")) return -1;
-    return seam_end(m, m->pf_logits, logits_cf, sizeof(float) * (size_t)m->cfg.vocab * seq, seq) ? 0 : -1;
+    return seam_end(m, seq, {{logits_cf, m->pf_logits, (size_t)m->cfg.vocab * seq}}) ? 0 : -1;
 }
 
 int sh_matmul_vocab_seq(const float *embed, const float *x_cf, int32_t vocab, int32_t dim,

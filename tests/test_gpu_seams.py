@@ -178,3 +178,20 @@ def test_conv_eval_matches_linear_cf(gpu):
     assert got.shape == (s, out_dim) and rel_err(got, want) <= 1e-5
     np.testing.assert_array_equal(conv.eval(x), got)   # a compiled kernel is reusable
     conv.close()
+
+
+def test_taps_device_time_leaves_the_host_copies_out(gpu):
+    """gpu_ms of a call with its taps (69 MB of them: 1.3 ms over PCIe at its best, against 0.25 ms
+    of kernels without them) covers the kernels, not the copies to the host; the least of five."""
+    cfg = sh.make_config(n_layers=1, max_seq=2000)
+    m, _, ow = build(cfg, sh.SH_DTYPE_F16, 61)
+    x = embed_cf(ow, sh.synth_tokens(2000, 62, cfg.vocab))
+    plain, taps = [], []
+    for _ in range(5):
+        m.layer_forward_cf(0, x)
+        plain.append(m.stats()["gpu_ms"])
+        m.layer_forward_cf_taps(0, x)
+        taps.append(m.stats()["gpu_ms"])
+    m.close()
+    print(f"{min(plain):.3f} ms, with taps {min(taps):.3f}")
+    assert min(plain) < min(taps) <= 4 * min(plain)
