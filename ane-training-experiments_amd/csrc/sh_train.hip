@@ -1486,9 +1486,11 @@ struct sh_trainer {
     };
     std::vector<Layer> lc;
     float *xL, *xnf, *rfin, *logits, *dy, *gatt, *ggate, *stats, *dlc, *gc, *loss, *cos_t, *sin_t;
-    // the backward's values that the side stream reads as well, each layer its own (dcur[l]: the
-    // gradient of layer l's input, dcur[L] the last layer's output's)
+    // the backward's values that the side stream reads as well (dcur[l]: the gradient of layer l's
+    // input, dcur[L] the last layer's output's): each layer's own, or, `turns` given, dcur three
+    // deep and the others two, layers of one parity taking turns
     std::vector<float *> dcur, gx2, gxf, gxa, dh13, dqkv;
+    bool turns;
     double *row_loss, *sq_part;
     int *row_valid;
     int32_t *ids, *in_ids, *in_off, *in_occ;   // compact target ids; input ids' positions
@@ -1502,9 +1504,10 @@ struct sh_trainer {
     hipEvent_t ev0, ev1;
     // Weight gradients and, where nothing has to see all of them first, Adam run here beside the
     // backward's chain on `stream`. ev_fork: what the chain has finished; ev_join: what the side
-    // stream has; ev_embed: the classifier's part of the embedding gradient.
+    // stream has; ev_embed: the classifier's part of the embedding gradient; ev_free: the side
+    // stream's reads of a layer's values, by layer parity (`turns`).
     hipStream_t side;
-    hipEvent_t ev_fork, ev_join, ev_embed;
+    hipEvent_t ev_fork, ev_join, ev_embed, ev_free[2];
     bool uploaded_globals;
     std::vector<bool> uploaded;
 };
@@ -1516,6 +1519,12 @@ constexpr int kSqParts = 1024;
 // Workgroups of a layer's Adam pass on the side stream: enough to keep up with the chain, few
 // enough to leave it the memory (a Stories110M step: 64 4.27 ms, 128 3.93, 256 3.86, 512 3.91).
 constexpr unsigned kSideAdamBlocks = 256;
+// The backward's values of all layers, 4 S L (7 D + 2 F) bytes, are each layer's own up to this much
+// (Stories110M: 116 MB at 256 positions, 233 at 512). Beyond it layers take turns: 1.9 GB at 4096
+// positions would be three quarters of what the forward keeps once more, and what waiting costs
+// is little beside a long window's layer (a step at 1024 positions 11.16 -> 11.22 ms, at 2048 22.38
+// -> 22.39).
+constexpr size_t kOwnBytes = 256u << 20;
 
 unsigned blocks_for(size_t n) { return (unsigned)std::min<size_t>((n + 255) / 256, 8192); }
 
@@ -1715,6 +1724,7 @@ hipError_t tr_forward_head(sh_trainer *T, int U, float loss_scale, bool acc) {
 // layer, and the values both streams read are each layer's own, so the chain never waits for the
 // side stream: with two forks and buffers by layer parity each layer's wait held the chain for
 // 20 us of event handling, though what it waited for was long done (eight steps 31.6 -> 30.75 ms).
+// Only where the values of all layers would take too much (kOwnBytes) do layers take turns.
 hipError_t tr_backward(sh_trainer *T, int n_in, bool acc, const AdamStep *adam) {
     hipStream_t s = T->stream, sd = T->side;
     const int S = T->S, D = T->D, F = T->F, hd = T->hd;
@@ -1724,6 +1734,8 @@ hipError_t tr_backward(sh_trainer *T, int n_in, bool acc, const AdamStep *adam) 
         sh_trainer::Layer &C = T->lc[l];
         float *dcur = T->dcur[l + 1], *dnext = T->dcur[l], *gx2 = T->gx2[l], *dh13 = T->dh13[l], *dqkv = T->dqkv[l],
               *gxf = T->gxf[l], *gxa = T->gxa[l];
+        // layer l + 2's weight gradients read the values of this parity (and its dcur this layer's dnext)
+        if (T->turns && l + 2 < T->L && (e = hipStreamWaitEvent(s, T->ev_free[l & 1], 0))) return e;
         // FFN: ggate = dout . W2 with dout = alpha dcur (the scale applied to the product),
         // (dh1, dh3), gxn = [dh1|dh3] . [W1;W3], RMS backward
         PartIn hg{}, hn{};   // split products' partials for the row kernels below
@@ -1800,6 +1812,7 @@ hipError_t tr_backward(sh_trainer *T, int n_in, bool acc, const AdamStep *adam) 
             return e;
         if ((e = sgemm_grad<false, false>(sd, dqkv, 3 * D, C.xn, D, T->g + T->o_qkv[l], D, 3 * D, D, S, acc)))
             return e;
+        if (T->turns && (e = hipEventRecord(T->ev_free[l & 1], sd))) return e;
         if (adam) launch_adam(T, T->o_qkv[l], (l + 1 < T->L ? T->o_qkv[l + 1] : T->o_embed) - T->o_qkv[l], *adam, sd, kSideAdamBlocks);
     }
     // the classifier's embedding gradient (the side stream's first work) comes before the inputs'
@@ -2043,10 +2056,12 @@ sh_trainer *sh_trainer_create(const sh_config *cfg, const sh_train_options *opt_
         lo[l].x2n = take(4 * S * D); lo[l].rf = take(4 * S); lo[l].h13 = take(4 * S * 2 * F);
         lo[l].gate = take(4 * S * F);
     }
+    T->turns = 4 * S * T->L * (7 * D + 2 * F) > kOwnBytes;
+    const size_t nd = T->turns ? std::min(3, T->L + 1) : T->L + 1, nb = T->turns ? std::min(2, T->L) : T->L;
     const size_t o_xL = take(4 * S * D), o_xnf = take(4 * S * D), o_rfin = take(4 * S), o_lg = take(4 * S * V),
-                 o_dy = take(4 * S * D), o_dcur = take(4 * (T->L + 1) * S * D), o_gx2 = take(4 * T->L * S * D),
-                 o_gxn = take(4 * 2 * T->L * S * D), o_gatt = take(4 * S * D), o_ggate = take(4 * S * F),
-                 o_dh13 = take(4 * T->L * S * 2 * F), o_dqkv = take(4 * T->L * S * 3 * D), o_stats = take(4 * 3 * T->H * S * T->L),
+                 o_dy = take(4 * S * D), o_dcur = take(4 * nd * S * D), o_gx2 = take(4 * nb * S * D),
+                 o_gxn = take(4 * 2 * nb * S * D), o_gatt = take(4 * S * D), o_ggate = take(4 * S * F),
+                 o_dh13 = take(4 * nb * S * 2 * F), o_dqkv = take(4 * nb * S * 3 * D), o_stats = take(4 * 3 * T->H * S * T->L),
                  o_dlc = take(4 * S * T->ldc_u), o_gc = take(4 * S * D), o_loss = take(16),
                  o_cos = take(4 * S * (T->hd / 2)), o_sin = take(4 * S * (T->hd / 2)), o_rl = take(8 * S),
                  o_sq = take(8 * kSqParts), o_rv = take(4 * S), o_ids = take(4 * S), o_ti = take(2 * S),
@@ -2061,7 +2076,7 @@ sh_trainer *sh_trainer_create(const sh_config *cfg, const sh_train_options *opt_
               hip_ok(hipMalloc(&T->act, a), "hipMalloc activations") &&
               hip_ok(hipMemset(T->p, 0, 4 * T->n_all), "clear") && hip_ok(hipMemset(T->g, 0, 4 * T->n_all), "clear") &&
               hip_ok(hipMemset(T->m, 0, 4 * T->n_all), "clear") && hip_ok(hipMemset(T->v, 0, 4 * T->n_all), "clear");
-    for (hipEvent_t *ev : {&T->ev_fork, &T->ev_join, &T->ev_embed})
+    for (hipEvent_t *ev : {&T->ev_fork, &T->ev_join, &T->ev_embed, &T->ev_free[0], &T->ev_free[1]})
         ok = ok && hip_ok(hipEventCreateWithFlags(ev, hipEventDisableTiming), "event");
     if (!ok) {
         sh_trainer_destroy(T);
@@ -2079,15 +2094,15 @@ sh_trainer *sh_trainer_create(const sh_config *cfg, const sh_train_options *opt_
     T->xL = (float *)(A + o_xL); T->xnf = (float *)(A + o_xnf); T->rfin = (float *)(A + o_rfin);
     T->logits = (float *)(A + o_lg); T->dy = (float *)(A + o_dy); T->gatt = (float *)(A + o_gatt);
     T->ggate = (float *)(A + o_ggate);
-    for (int l = 0; l < T->L; l++) {
-        T->dcur.push_back((float *)(A + o_dcur) + l * S * D);
-        T->gx2.push_back((float *)(A + o_gx2) + l * S * D);
-        T->gxf.push_back((float *)(A + o_gxn) + 2 * l * S * D);
-        T->gxa.push_back((float *)(A + o_gxn) + (2 * l + 1) * S * D);
-        T->dh13.push_back((float *)(A + o_dh13) + l * S * 2 * F);
-        T->dqkv.push_back((float *)(A + o_dqkv) + l * S * 3 * D);
+    for (size_t l = 0; l <= (size_t)T->L; l++) T->dcur.push_back((float *)(A + o_dcur) + l % nd * S * D);
+    for (size_t l = 0; l < (size_t)T->L; l++) {
+        const size_t i = l % nb;
+        T->gx2.push_back((float *)(A + o_gx2) + i * S * D);
+        T->gxf.push_back((float *)(A + o_gxn) + 2 * i * S * D);
+        T->gxa.push_back((float *)(A + o_gxn) + (2 * i + 1) * S * D);
+        T->dh13.push_back((float *)(A + o_dh13) + i * S * 2 * F);
+        T->dqkv.push_back((float *)(A + o_dqkv) + i * S * 3 * D);
     }
-    T->dcur.push_back((float *)(A + o_dcur) + T->L * S * D);
     T->stats = (float *)(A + o_stats); T->dlc = (float *)(A + o_dlc); T->gc = (float *)(A + o_gc);
     T->loss = (float *)(A + o_loss); T->cos_t = (float *)(A + o_cos); T->sin_t = (float *)(A + o_sin);
     T->row_loss = (double *)(A + o_rl); T->sq_part = (double *)(A + o_sq); T->row_valid = (int *)(A + o_rv);
@@ -2261,7 +2276,7 @@ void sh_trainer_destroy(sh_trainer *T) {
     (void)hipFree(T->act);
     if (T->stream) (void)hipStreamDestroy(T->stream);
     if (T->side) (void)hipStreamDestroy(T->side);
-    for (hipEvent_t ev : {T->ev0, T->ev1, T->ev_fork, T->ev_join, T->ev_embed})
+    for (hipEvent_t ev : {T->ev0, T->ev1, T->ev_fork, T->ev_join, T->ev_embed, T->ev_free[0], T->ev_free[1]})
         if (ev) (void)hipEventDestroy(ev);
     delete T;
 }
