@@ -2,7 +2,10 @@
 wrong: segments one off a 64-key block and a 128-query tile, sequences of rows that do not start
 on a tile, head dims 64 and 128, fp16 and bf16, one to eight q heads' worth of grid at the line
 that its dispatch draws. Batched prompts against the oracle's single-sequence decoder: the first
-new token's logits of every sequence within 2e-2, as everywhere (measured about 1e-3)."""
+new token's logits of three sequences, 2-norm of the difference over that of the logits. A key or value
+of the cache that is rounded the other way makes up to 4.5e-4 in bf16 and 5.7e-5 in fp16 (an fp32 cache:
+8e-6); dropping the lo plane of Q, P or the output makes 8.7e-4 to 2.8e-3 in bf16 and 1.1e-4 to 3.5e-4 in
+fp16, leaving out one key of the last row 0.05 to 0.1 (the float64 model with the mistake planted)."""
 import numpy as np
 import pytest
 
@@ -42,6 +45,6 @@ def test_prompt_attention(gpu, shape, dtype, kv, seqs, seg):
         ref.reset()
         for p in range(seg + 1):
             want = ref.forward_one(int(prompts[b, p]), p)
-        err = float(np.max(np.abs(got[0, k] - want)))
-        print(f"sequence {b}: max-abs {err:.2e} (max |logit| {np.abs(want).max():.2f})")
-        assert err <= 2e-2
+        err = float(np.linalg.norm(got[0, k].astype(np.float64) - want) / np.linalg.norm(want))
+        print(f"sequence {b}: {err:.2e}")
+        assert err <= {sh.SH_KV_BF16: 8e-4, sh.SH_KV_F16: 1e-4, sh.SH_KV_F32: 3e-5}[kv]

@@ -1,15 +1,20 @@
 """The 16-bit GEMM's tile shapes at their edges (k_linear_few, k_gemm_pipe and k_gemm_ring,
-chosen by linear_few and gemm_plan): row counts one off a tile, K ranges of one step, of an odd number of steps and of
-an uneven split, N that fits only the narrower tiles, and each epilogue, through the entry points.
+chosen by linear_few and gemm_plan, whose choice each case names): row counts one off a tile, K
+ranges of one step, of an odd number of steps and of an uneven split, N that fits only the
+narrower tiles, and each epilogue, through the entry points.
 
-ConvEval (fp16 weights, activations as hi/lo pairs of fp16) against float64: each output's error
+ConvEval (fp16 weights, activations as hi/lo pairs of fp16) against float64. Each output's error
 is at most (2^-21 + (K + 2) * 2^-23) * sum |w x|, the pair's 22 bits and two fp32 roundings per
-element of the sum. The layer seam and EvalLogits against the oracle keep the bars of their own
-tests."""
+element of the sum. And in every block of 16 x 16 results, the least that a wave computes, the root mean
+square of the error is at most 4 * (2^-24 * sqrt(K / 16 + 8) + 2^-22) of that of all results: a sum of K / 32
+products of each plane, rounded each time, and the pair's rounding. One fp16 plane in the place of the
+pair exceeds that in every case (checked on the CPU). The layer seam and EvalLogits against the
+oracle keep the bars of their own tests."""
 import numpy as np
 import pytest
 
 import oracle
+import plan
 import stories_hip as sh
 from helpers import tiny_config, tiny_gqa_config
 from test_zz_no_alloc import Hip
@@ -18,18 +23,31 @@ from test_gpu_seams import THREADS, build, embed_cf, rel_err
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("s,in_dim,out_dim", [
-    (1, 2048, 4096), (15, 4096, 64), (16, 1056, 192), (17, 1536, 448),   # one launch: a few rows
-    (31, 224, 4096), (128, 768, 768), (127, 32, 1024),
-    (1, 32, 64), (3, 64, 64), (65, 96, 192),         # K of one to three steps: fewer than the ring's slots
-    (31, 1056, 64), (33, 1056, 1088), (64, 416, 448),  # 32 x 64 tiles: uneven K ranges, K % 64 == 32
-    (65, 192, 768), (129, 768, 768),                 # the pipelined 32 x 32 tiles, split and unsplit
-    (1091, 2048, 768),                               # 64 x 64 tiles
-    (513, 512, 4096), (577, 768, 2304),              # 64 x 128 tiles
-    (127, 768, 32000), (1023, 1024, 3072), (641, 1024, 4096),   # 128 x 128 tiles
-    (193, 768, 32000), (2049, 512, 6144),            # 128 x 256 tiles
+def block_rms(e):
+    """Root mean squares of the 16 x 16 blocks of e."""
+    r, c = np.arange(0, e.shape[0], 16), np.arange(0, e.shape[1], 16)
+    n = np.add.reduceat(np.add.reduceat(np.ones_like(e), r, 0), c, 1)
+    return np.sqrt(np.add.reduceat(np.add.reduceat(e * e, r, 0), c, 1) / n)
+
+
+@pytest.mark.parametrize("kernel,s,in_dim,out_dim", [
+    ("few", 1, 2048, 4096), ("few", 15, 4096, 64), ("few", 16, 1056, 192), ("few", 17, 1536, 448),   # one launch
+    ("few", 31, 224, 4096), ("few", 128, 768, 768), ("few", 127, 32, 1024), ("few", 1, 32, 64), ("few", 3, 64, 64),
+    ("few", 65, 96, 192), ("few", 31, 1056, 64), ("few", 33, 1056, 1088), ("few", 64, 416, 448),
+    ("few", 65, 192, 768), ("few", 129, 768, 768),
+    # K of one to three steps, fewer than the ring's slots
+    ("ring32x64/1", 300, 32, 1024), ("ring32x64/1", 299, 96, 1024), ("ring64x64/1", 301, 32, 6144),
+    ("ring64x64/1", 193, 96, 4096), ("ring64x128/1", 1501, 32, 4096), ("ring64x128/1", 531, 64, 6144),
+    # uneven K ranges, K % 64 == 32
+    ("ring32x64/4", 33, 1568, 1088), ("ring32x64/4", 200, 1568, 256), ("ring32x64/4", 33, 2016, 192),
+    # the pipelined 32 x 32 tiles, split and unsplit
+    ("pipe32/4", 65, 2048, 192), ("pipe32/2", 257, 768, 768), ("pipe32/1", 700, 256, 1024),
+    ("ring64x64/1", 1091, 2048, 768), ("ring64x128/1", 513, 512, 4096), ("ring64x128/1", 577, 768, 2304),
+    ("ring128x128/1", 127, 768, 32000), ("ring128x128/1", 1023, 1024, 3072), ("ring128x128/1", 641, 1024, 4096),
+    ("ring128x128/1", 193, 768, 32000), ("ring128x256/1", 2049, 512, 6144),
 ])
-def test_conv_eval_tile_shapes(gpu, s, in_dim, out_dim):
+def test_conv_eval_tile_shapes(gpu, kernel, s, in_dim, out_dim):
+    assert plan.conv_kernel(s, in_dim, out_dim) == kernel
     rng = np.random.default_rng(s + in_dim + out_dim)
     w = (rng.standard_normal((out_dim, in_dim), np.float32) * 0.05).astype(np.float32)
     x = rng.standard_normal((s, in_dim), np.float32)
@@ -40,8 +58,15 @@ def test_conv_eval_tile_shapes(gpu, s, in_dim, out_dim):
     want = x.astype(np.float64) @ w16.T
     bound = (2.0 ** -21 + (in_dim + 2) * 2.0 ** -23) * (np.abs(x).astype(np.float64) @ np.abs(w16).T)
     worst = float(np.max(np.abs(got - want) / bound))
-    print(f"{s} x {out_dim} x {in_dim}: {worst:.2e} of the bound")
-    assert worst <= 1.0
+    rms = float(np.sqrt(np.mean(want * want)))
+    block = float(block_rms(got - want).max()) / rms
+    bar = 4 * (2.0 ** -24 * np.sqrt(in_dim / 16 + 8) + 2.0 ** -22)
+    n = min(s, 16)
+    plane = x[:n].astype(np.float16).astype(np.float64) @ w16.T - want[:n]
+    print(f"{s} x {out_dim} x {in_dim}: {worst:.2e} of the bound, blocks {block / bar:.2f} of theirs, "
+          f"one plane {block_rms(plane).min() / rms / bar:.1f}")
+    assert worst <= 1.0 and block <= bar
+    assert block_rms(plane).min() / rms > bar
 
 
 @pytest.mark.parametrize("s,in_dim,out_dim", [(5, 256, 128), (40, 2048, 192), (700, 512, 1024)])
@@ -72,13 +97,20 @@ def test_conv_eval_noalloc_unaligned_buffers(gpu, s, in_dim, out_dim, off):
         conv.close()
 
 
-@pytest.mark.parametrize("make_cfg,dtype,seq", [
-    # every layer product on the ring: residual (N = 768) and gate (N = 4096 and 1536) epilogues
-    (lambda: tiny_config(dim=768, hidden=2048, n_heads=12, n_kv_heads=12, head_dim=64, max_seq=1100), sh.SH_DTYPE_F16, 1091),
-    (lambda: tiny_gqa_config(dim=256, hidden=768, n_heads=8, n_kv_heads=4, max_seq=700), sh.SH_DTYPE_BF16, 641),
+# the kernels of q|k|v, Wo (residual), W1|W3 (gate) and W2 (residual)
+@pytest.mark.parametrize("make_cfg,dtype,seq,kernels", [
+    (lambda: tiny_config(dim=768, hidden=2048, n_heads=12, n_kv_heads=12, head_dim=64, max_seq=1100), sh.SH_DTYPE_F16, 1091,
+     "ring128x128 ring64x64 ring64x128 ring64x64"),
+    (lambda: tiny_gqa_config(dim=256, hidden=768, n_heads=8, n_kv_heads=4, max_seq=700), sh.SH_DTYPE_BF16, 641,
+     "pipe32 pipe32 pipe32 pipe32"),
+    (lambda: tiny_gqa_config(dim=512, hidden=3072, n_heads=16, n_kv_heads=8, max_seq=1100), sh.SH_DTYPE_BF16, 1091,
+     "ring64x128 pipe32 ring128x256 pipe32"),
 ])
-def test_layer_forward_on_ring_tiles(gpu, make_cfg, dtype, seq):
+def test_layer_forward_on_ring_tiles(gpu, make_cfg, dtype, seq, kernels):
     cfg = make_cfg()
+    D, F, Q = cfg.dim, cfg.hidden, cfg.qdim
+    products = [(seq, Q + 2 * cfg.kvdim, D, 0), (seq, D, Q, 0), (seq, 2 * F, D, 0), (seq, D, F, 0)]
+    assert [p.kind for p in plan.plans(products)] == kernels.split()
     m, ocfg, ow = build(cfg, dtype, 71, std=0.03)
     x = embed_cf(ow, sh.synth_tokens(seq, 72, cfg.vocab))
     got = m.layer_forward_cf(0, x)
@@ -89,12 +121,12 @@ def test_layer_forward_on_ring_tiles(gpu, make_cfg, dtype, seq):
     assert err <= 1e-4
 
 
-@pytest.mark.parametrize("dtype,seq,vocab", [
-    (sh.SH_DTYPE_F16, 47, 32000), (sh.SH_DTYPE_F16, 190, 32064),   # 64 x 64 tiles
-    (sh.SH_DTYPE_F16, 188, 16384),                                 # 128 x 128 tiles, one plane
-    (sh.SH_DTYPE_BF16, 189, 16384)])                               # 64 x 128 tiles
-def test_eval_logits_on_ring_tiles(gpu, dtype, seq, vocab):
-    """Channel-first logits of row counts that are and are not multiples of four."""
+@pytest.mark.parametrize("dtype,seq,vocab,kernel", [
+    (sh.SH_DTYPE_F16, 47, 32000, "ring64x64"), (sh.SH_DTYPE_F16, 190, 32064, "ring64x64"),
+    (sh.SH_DTYPE_F16, 188, 16384, "ring128x128"), (sh.SH_DTYPE_BF16, 189, 16384, "ring64x128")])
+def test_eval_logits_on_ring_tiles(gpu, dtype, seq, vocab, kernel):
+    """Channel-first logits of row counts that are and are not multiples of four; fp16 in one plane."""
+    assert plan.plans([(seq, vocab, 256, dtype == sh.SH_DTYPE_F16)])[0].kind == kernel
     cfg = tiny_config(dim=256, hidden=512, n_heads=4, n_kv_heads=4, head_dim=64, vocab=vocab, max_seq=256)
     m, ocfg, ow = build(cfg, dtype, 81)
     toks = sh.synth_tokens(seq, 82, cfg.vocab)
