@@ -1720,7 +1720,7 @@ hipError_t tr_forward_head(sh_trainer *T, int U, float loss_scale, bool acc) {
 // Only the input gradients form a chain, of small products and row kernels that leave most of
 // the chip idle (122 us per Stories110M layer at S = 256); the weight gradients (64 us) and, with
 // `adam` given, the layer's Adam pass (50 us, bound by memory) go to the side stream, each layer's
-// as soon as the chain no longer reads its weights. One step: 4.23 -> 3.84 ms. One fork per
+// as soon as the chain no longer reads its weights. One step: 4.23 -> 3.86 ms. One fork per
 // layer, and the values both streams read are each layer's own, so the chain never waits for the
 // side stream: with two forks and buffers by layer parity each layer's wait held the chain for
 // 20 us of event handling, though what it waited for was long done (eight steps 31.6 -> 30.75 ms).
@@ -1829,7 +1829,7 @@ hipError_t tr_backward(sh_trainer *T, int n_in, bool acc, const AdamStep *adam) 
 // :149-181) and Adam at 1-based step step_t (:838-842); k_tr_adam leaves the applied gradients
 // in the arena. layers_done: the layers' matrices have theirs on the side stream (tr_backward), and
 // the embedding's pass, a fifth of them all, runs beside the last of it, on as few workgroups (on
-// 4096 it held the side stream up for as long as it saved): eight steps 30.0 -> 29.6 ms.
+// 4096 it held the side stream up for as long as it saved): eight steps 30.0 -> 29.7 ms.
 hipError_t tr_apply(sh_trainer *T, float inv, int step_t, bool layers_done) {
     hipStream_t s = T->stream;
     hipError_t e;
