@@ -33,9 +33,10 @@ inline bool gemm_one_plane(int M, int N, int K) { return gemm_big(M, N) ? K % 12
 enum { GK_PIPE32 = 0, GK_RING128x256, GK_RING128x128, GK_RING64x128, GK_RING64x64, GK_RING32x64 };
 struct GemmPlan {
     int kind, ranges, kc;
+    int run;   // K steps of 32 that are added into one sum before it joins the total; 0: all of them
 };
-inline GemmPlan gemm_plan(int M, int N, int K, bool one_plane) {
-    GemmPlan p{GK_RING64x64, 1, K};
+inline GemmPlan gemm_plan(int M, int N, int K, bool one_plane, bool bf16) {
+    GemmPlan p{GK_RING64x64, 1, K, 0};
     float best = INFINITY;
     const auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * (N / bn); };
     const auto ring = [&](int kind, int bm, int bn, float step, float base) {
@@ -46,11 +47,17 @@ inline GemmPlan gemm_plan(int M, int N, int K, bool one_plane) {
             p.kind = kind;
         }
     };
+    // The products that used to be split into K ranges for want of tiles, and so had short sums: as
+    // fp16 pairs they keep them, 512 of K at a time. 1100 x 1024 x 2048: relative error 1.6e-7, against
+    // 2.9e-7 in one sum and 2.2e-7 in the four ranges before (29.8 -> 31.9 us); 1024 x 768 x 768 12.5 ->
+    // 13.1 us, 25.0 in ranges. A bf16 pair's own 1e-6 hides the sum's error.
+    const bool runs = !one_plane && !bf16 && gemm_big(M, N) && tiles(128, 128) <= 384;
+    if (runs) p.run = 16;
     // These tiles' registers hold one sum per result, so a pair's lo products are added into the hi
     // products' sums: large products only, which never had two. Others keep sums of their own, at 64.7
     // us against 62.3 and an error of 2.9e-7 against 4.1e-7 for 700 x 6144 x 2048 (193 x 32000 x 768:
     // 37.0 against 34.4 us, 1.9e-7 against 2.6e-7).
-    if (one_plane || gemm_big(M, N))
+    if (one_plane || (gemm_big(M, N) && !runs))
         ring(GK_RING128x256, 128, 256, one_plane ? 0.40f : 0.75f, one_plane ? 6.3f : 7.0f);
     ring(GK_RING128x128, 128, 128, one_plane ? 0.26f : 0.48f, one_plane ? 4.0f : 4.5f);
     if (!one_plane) ring(GK_RING64x128, 64, 128, 0.28f, 3.0f);
@@ -66,7 +73,7 @@ inline GemmPlan gemm_plan(int M, int N, int K, bool one_plane) {
     }
     const int per = (steps + ranges - 1) / ranges;   // K steps per range
     if (2.3f + per * std::max(t32 * ranges, 300) * (one_plane ? 4.1e-4f : 6.3e-4f) < best)
-        p = GemmPlan{pipe ? GK_PIPE32 : GK_RING32x64, (steps + per - 1) / per, per * unit};
+        p = GemmPlan{pipe ? GK_PIPE32 : GK_RING32x64, (steps + per - 1) / per, per * unit, p.run};
     return p;
 }
 

@@ -8,16 +8,16 @@ from collections import namedtuple
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 KINDS = ("pipe32", "ring128x256", "ring128x128", "ring64x128", "ring64x64", "ring32x64")
-Plan = namedtuple("Plan", "kind ranges kc one_plane_ok few")
+Plan = namedtuple("Plan", "kind ranges kc run one_plane_ok few")
 
 SOURCE = r"""
 #include "sh_gemm_plan.hpp"
 #include <stdio.h>
 int main() {
-    int m, n, k, one;
-    while (scanf("%d %d %d %d", &m, &n, &k, &one) == 4) {
-        const sh::GemmPlan p = sh::gemm_plan(m, n, k, one);
-        printf("%d %d %d %d %d\n", p.kind, p.ranges, p.kc, sh::gemm_one_plane(m, n, k), sh::linear_few(m, n, k, false));
+    int m, n, k, one, bf;
+    while (scanf("%d %d %d %d %d", &m, &n, &k, &one, &bf) == 5) {
+        const sh::GemmPlan p = sh::gemm_plan(m, n, k, one, bf);
+        printf("%d %d %d %d %d %d\n", p.kind, p.ranges, p.kc, p.run, sh::gemm_one_plane(m, n, k), sh::linear_few(m, n, k, false));
     }
 }
 """
@@ -36,15 +36,15 @@ def _program():
 
 
 def plans(products):
-    """Plan of each (M, N, K, one_plane)."""
-    text = "\n".join("%d %d %d %d" % tuple(p) for p in products)
+    """Plan of each (M, N, K, one_plane[, bf16])."""
+    text = "\n".join("%d %d %d %d %d" % (*p, 0)[:5] for p in products)
     out = subprocess.run([_program()[0]], input=text, capture_output=True, text=True, check=True).stdout
     rows = [[int(v) for v in line.split()] for line in out.splitlines()]
     assert len(rows) == len(products)
-    return [Plan(KINDS[r[0]], r[1], r[2], bool(r[3]), bool(r[4])) for r in rows]
+    return [Plan(KINDS[r[0]], *r[1:4], bool(r[4]), bool(r[5])) for r in rows]
 
 
 def conv_kernel(s, in_dim, out_dim):
     """The kernel of a ConvEval: "few", or the plan's kind with its K ranges."""
     p = plans([(s, out_dim, in_dim, 0)])[0]
-    return "few" if p.few else "%s/%d" % (p.kind, p.ranges)
+    return "few" if p.few else "%s/%d%s" % (p.kind, p.ranges, " in runs" if p.run else "")

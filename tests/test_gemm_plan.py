@@ -28,3 +28,21 @@ def test_pairs_keep_sums_of_their_own():
         assert large or p.kind != "ring128x256", (m, n, k)
     # sizes that took them: two rounds of the next smaller tile
     assert {p.kind for p in plans([(193, 32000, 768, 0), (700, 6144, 2048, 0), (1000, 6144, 2048, 0)])} == {"ring128x128", "ring64x128"}
+
+
+def test_sums_no_longer_than_those_of_the_ranges_before():
+    """Large fp16 pairs of at most 384 tiles of 128 x 128 were split into K ranges, each with one sum of
+    2 K / 32 / ranges products. Their sums have at most as many now: 16 steps of one plane, or all of a
+    shorter K, then one addition per run."""
+    products = [(m, n, k, 0) for m, n, k in itertools.product(ROWS, (*COLS, 6144), (*WIDTHS, 544, 1568)) if m >= 256]
+    seen = 0
+    for (m, n, k, _), p in zip(products, plans(products)):
+        large = (m >= 1024 or n >= 16384) and n % 128 == 0
+        tiles = -(-m // 128) * (n // 128)
+        ranges = max((r for r in (2, 3, 4) if k % (32 * r) == 0 and k // r >= 256 and tiles * r <= 768), default=1)
+        if not large or tiles >= 512 or ranges == 1:
+            continue
+        seen += 1
+        own = min(p.kc // 32, p.run or k)
+        assert p.kind != "ring128x256" and own <= 2 * k // 32 // ranges, (m, n, k)
+    assert seen > 100

@@ -30,6 +30,10 @@ def block_rms(e):
     return np.sqrt(np.add.reduceat(np.add.reduceat(e * e, r, 0), c, 1) / n)
 
 
+def block_bar(K):
+    return 4 * (2.0 ** -24 * np.sqrt(K / 16 + 8) + 2.0 ** -22)
+
+
 @pytest.mark.parametrize("kernel,s,in_dim,out_dim", [
     ("few", 1, 2048, 4096), ("few", 15, 4096, 64), ("few", 16, 1056, 192), ("few", 17, 1536, 448),   # one launch
     ("few", 31, 224, 4096), ("few", 128, 768, 768), ("few", 127, 32, 1024), ("few", 1, 32, 64), ("few", 3, 64, 64),
@@ -37,12 +41,15 @@ def block_rms(e):
     ("few", 65, 192, 768), ("few", 129, 768, 768),
     # K of one to three steps, fewer than the ring's slots
     ("ring32x64/1", 300, 32, 1024), ("ring32x64/1", 299, 96, 1024), ("ring64x64/1", 301, 32, 6144),
-    ("ring64x64/1", 193, 96, 4096), ("ring64x128/1", 1501, 32, 4096), ("ring64x128/1", 531, 64, 6144),
+    ("ring64x64/1", 193, 96, 4096), ("ring64x128/1 in runs", 1501, 32, 4096), ("ring64x128/1", 531, 64, 6144),
     # uneven K ranges, K % 64 == 32
     ("ring32x64/4", 33, 1568, 1088), ("ring32x64/4", 200, 1568, 256), ("ring32x64/4", 33, 2016, 192),
     # the pipelined 32 x 32 tiles, split and unsplit
     ("pipe32/4", 65, 2048, 192), ("pipe32/2", 257, 768, 768), ("pipe32/1", 700, 256, 1024),
-    ("ring64x64/1", 1091, 2048, 768), ("ring64x128/1", 513, 512, 4096), ("ring64x128/1", 577, 768, 2304),
+    # sums of 512 of K at a time: an uneven last run, none, every kernel that has them
+    ("pipe32/1 in runs", 1024, 768, 768), ("ring64x64/1 in runs", 1091, 2048, 768), ("ring128x128/1 in runs", 1091, 768, 2048),
+    ("ring64x128/1 in runs", 1501, 1536, 1024), ("ring32x64/2 in runs", 1024, 1568, 512),
+    ("ring64x128/1", 513, 512, 4096), ("ring64x128/1", 577, 768, 2304),
     ("ring128x128/1", 127, 768, 32000), ("ring128x128/1", 1023, 1024, 3072), ("ring128x128/1", 641, 1024, 4096),
     ("ring128x128/1", 193, 768, 32000), ("ring128x256/1", 2049, 512, 6144),
 ])
@@ -60,13 +67,30 @@ def test_conv_eval_tile_shapes(gpu, kernel, s, in_dim, out_dim):
     worst = float(np.max(np.abs(got - want) / bound))
     rms = float(np.sqrt(np.mean(want * want)))
     block = float(block_rms(got - want).max()) / rms
-    bar = 4 * (2.0 ** -24 * np.sqrt(in_dim / 16 + 8) + 2.0 ** -22)
+    bar = block_bar(in_dim)
     n = min(s, 16)
     plane = x[:n].astype(np.float16).astype(np.float64) @ w16.T - want[:n]
     print(f"{s} x {out_dim} x {in_dim}: {worst:.2e} of the bound, blocks {block / bar:.2f} of theirs, "
           f"one plane {block_rms(plane).min() / rms / bar:.1f}")
     assert worst <= 1.0 and block <= bar
     assert block_rms(plane).min() / rms > bar
+
+
+@pytest.mark.parametrize("kernel,seq,dim,vocab", [
+    ("pipe32/1 in runs", 1100, 768, 512), ("ring64x128/1 in runs", 1030, 1056, 1024), ("ring128x128/1 in runs", 1030, 768, 2048),
+    ("ring64x64/1 in runs", 2001, 768, 512), ("ring32x64/2 in runs", 1030, 1056, 512)])
+def test_channel_first_product_in_runs(gpu, kernel, seq, dim, vocab):
+    """The same sums in channel-first logits (MatMulVocabSeq), by blocks as above."""
+    p = plan.plans([(seq, vocab, dim, 0)])[0]
+    assert "%s/%d in runs" % (p.kind, p.ranges) == kernel and p.run
+    rng = np.random.default_rng(seq + dim)
+    e = (rng.standard_normal((vocab, dim), np.float32) * 0.05).astype(np.float32)
+    x = rng.standard_normal((dim, seq), np.float32)
+    got = sh.matmul_vocab_seq(e, x)
+    want = e.astype(np.float16).astype(np.float64) @ x.astype(np.float64)
+    block = float(block_rms(got - want).max()) / float(np.sqrt(np.mean(want * want)))
+    print(f"{block / block_bar(dim):.2f} of the bar")
+    assert block <= block_bar(dim)
 
 
 @pytest.mark.parametrize("s,in_dim,out_dim", [(5, 256, 128), (40, 2048, 192), (700, 512, 1024)])
