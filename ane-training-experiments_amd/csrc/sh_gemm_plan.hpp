@@ -47,17 +47,18 @@ inline GemmPlan gemm_plan(int M, int N, int K, bool one_plane, bool bf16) {
             p.kind = kind;
         }
     };
-    // The products that used to be split into K ranges for want of tiles, and so had short sums: as
-    // fp16 pairs they keep them, 512 of K at a time. 1100 x 1024 x 2048: relative error 1.6e-7, against
-    // 2.9e-7 in one sum and 2.2e-7 in the four ranges before (29.8 -> 31.9 us); 1024 x 768 x 768 12.5 ->
-    // 13.1 us, 25.0 in ranges. A bf16 pair's own 1e-6 hides the sum's error.
-    const bool runs = !one_plane && !bf16 && gemm_big(M, N) && tiles(128, 128) <= 384;
-    if (runs) p.run = 16;
+    // For want of tiles some products were split into K ranges by the kernels before these (large ones,
+    // and those of K not a multiple of 64), each range with one sum of both planes' products.
+    const int t = gemm_big(M, N) ? tiles(128, 128) : tiles(64, 64);
+    int before = 1;
+    if (!one_plane && !bf16 && t < 512 && (gemm_big(M, N) || K % 64))
+        for (int r : {2, 3, 4})
+            if (K % (32 * r) == 0 && K / r >= 256 && t * r <= 768) before = r;
     // These tiles' registers hold one sum per result, so a pair's lo products are added into the hi
     // products' sums: large products only, which never had two. Others keep sums of their own, at 64.7
     // us against 62.3 and an error of 2.9e-7 against 4.1e-7 for 700 x 6144 x 2048 (193 x 32000 x 768:
     // 37.0 against 34.4 us, 1.9e-7 against 2.6e-7).
-    if (one_plane || (gemm_big(M, N) && !runs))
+    if (one_plane || (gemm_big(M, N) && before == 1))
         ring(GK_RING128x256, 128, 256, one_plane ? 0.40f : 0.75f, one_plane ? 6.3f : 7.0f);
     ring(GK_RING128x128, 128, 128, one_plane ? 0.26f : 0.48f, one_plane ? 4.0f : 4.5f);
     if (!one_plane) ring(GK_RING64x128, 64, 128, 0.28f, 3.0f);
@@ -73,7 +74,13 @@ inline GemmPlan gemm_plan(int M, int N, int K, bool one_plane, bool bf16) {
     }
     const int per = (steps + ranges - 1) / ranges;   // K steps per range
     if (2.3f + per * std::max(t32 * ranges, 300) * (one_plane ? 4.1e-4f : 6.3e-4f) < best)
-        p = GemmPlan{pipe ? GK_PIPE32 : GK_RING32x64, (steps + per - 1) / per, per * unit, p.run};
+        p = GemmPlan{pipe ? GK_PIPE32 : GK_RING32x64, (steps + per - 1) / per, per * unit, 0};
+    // As fp16 pairs such products keep sums no longer than those: where one plane's K steps are more, 512
+    // of K at a time. 1100 x 1024 x 2048: relative error 1.6e-7, against 2.9e-7 in one sum and 2.2e-7 in
+    // the four ranges before (29.8 -> 31.9 us); 1024 x 768 x 768 12.5 -> 13.1 us, 25.0 in ranges; 300 x
+    // 2560 x 2016 1.6e-7 against 2.9e-7 and 2.4e-7, 24.2 -> 27.2 us, 27.5 in ranges. A bf16 pair's own
+    // 1e-6 hides the sum's error.
+    if (before > 1 && p.kc / 32 > 2 * (K / 32) / before) p.run = 16;
     return p;
 }
 

@@ -31,18 +31,22 @@ def test_pairs_keep_sums_of_their_own():
 
 
 def test_sums_no_longer_than_those_of_the_ranges_before():
-    """Large fp16 pairs of at most 384 tiles of 128 x 128 were split into K ranges, each with one sum of
-    2 K / 32 / ranges products. Their sums have at most as many now: 16 steps of one plane, or all of a
-    shorter K, then one addition per run."""
-    products = [(m, n, k, 0) for m, n, k in itertools.product(ROWS, (*COLS, 6144), (*WIDTHS, 544, 1568)) if m >= 256]
-    seen = 0
+    """Large fp16 pairs of at most 384 tiles of 128 x 128, and others of K not a multiple of 64 and at most
+    256 tiles of 64 x 64, were split into K ranges, each with one sum of 2 K / 32 / ranges products. Their
+    sums have at most as many now: 16 steps of one plane, or all of a shorter K, then one addition per run."""
+    products = [(m, n, k, 0) for m, n, k in
+                itertools.product((*ROWS, 174, 300, 446), (*COLS, 2176, 3520, 6144), (*WIDTHS, 544, 1248, 1568, 1632, 2016, 2976))]
+    seen = {True: 0, False: 0}
     for (m, n, k, _), p in zip(products, plans(products)):
-        large = (m >= 1024 or n >= 16384) and n % 128 == 0
-        tiles = -(-m // 128) * (n // 128)
-        ranges = max((r for r in (2, 3, 4) if k % (32 * r) == 0 and k // r >= 256 and tiles * r <= 768), default=1)
-        if not large or tiles >= 512 or ranges == 1:
+        large = (m >= 1024 or (m >= 256 and n >= 16384)) and n % 128 == 0
+        if p.few or (not large and k % 64 == 0):
             continue
-        seen += 1
+        t = 128 if large else 64
+        tiles = -(-m // t) * (n // t)
+        ranges = max((r for r in (2, 3, 4) if k % (32 * r) == 0 and k // r >= 256 and tiles * r <= 768), default=1)
+        if tiles >= 512 or ranges == 1:
+            continue
+        seen[large] += 1
         own = min(p.kc // 32, p.run or k)
         assert p.kind != "ring128x256" and own <= 2 * k // 32 // ranges, (m, n, k)
-    assert seen > 100
+    assert min(seen.values()) > 50, seen

@@ -41,14 +41,15 @@ def block_bar(K):
     ("few", 65, 192, 768), ("few", 129, 768, 768),
     # K of one to three steps, fewer than the ring's slots
     ("ring32x64/1", 300, 32, 1024), ("ring32x64/1", 299, 96, 1024), ("ring64x64/1", 301, 32, 6144),
-    ("ring64x64/1", 193, 96, 4096), ("ring64x128/1 in runs", 1501, 32, 4096), ("ring64x128/1", 531, 64, 6144),
+    ("ring64x64/1", 193, 96, 4096), ("ring64x128/1", 1501, 32, 4096), ("ring64x128/1", 531, 64, 6144),
     # uneven K ranges, K % 64 == 32
     ("ring32x64/4", 33, 1568, 1088), ("ring32x64/4", 200, 1568, 256), ("ring32x64/4", 33, 2016, 192),
     # the pipelined 32 x 32 tiles, split and unsplit
     ("pipe32/4", 65, 2048, 192), ("pipe32/2", 257, 768, 768), ("pipe32/1", 700, 256, 1024),
     # sums of 512 of K at a time: an uneven last run, none, every kernel that has them
     ("pipe32/1 in runs", 1024, 768, 768), ("ring64x64/1 in runs", 1091, 2048, 768), ("ring128x128/1 in runs", 1091, 768, 2048),
-    ("ring64x128/1 in runs", 1501, 1536, 1024), ("ring32x64/2 in runs", 1024, 1568, 512),
+    ("ring64x128/1 in runs", 1501, 1536, 1024), ("ring32x64/2", 1024, 1568, 512),
+    ("ring64x64/1 in runs", 300, 2016, 2560), ("ring32x64/1 in runs", 190, 1632, 4096),
     ("ring64x128/1", 513, 512, 4096), ("ring64x128/1", 577, 768, 2304),
     ("ring128x128/1", 127, 768, 32000), ("ring128x128/1", 1023, 1024, 3072), ("ring128x128/1", 641, 1024, 4096),
     ("ring128x128/1", 193, 768, 32000), ("ring128x256/1", 2049, 512, 6144),
@@ -78,7 +79,7 @@ def test_conv_eval_tile_shapes(gpu, kernel, s, in_dim, out_dim):
 
 @pytest.mark.parametrize("kernel,seq,dim,vocab", [
     ("pipe32/1 in runs", 1100, 768, 512), ("ring64x128/1 in runs", 1030, 1056, 1024), ("ring128x128/1 in runs", 1030, 768, 2048),
-    ("ring64x64/1 in runs", 2001, 768, 512), ("ring32x64/2 in runs", 1030, 1056, 512)])
+    ("ring64x64/1 in runs", 2001, 768, 512), ("ring32x64/1 in runs", 190, 1632, 4096)])
 def test_channel_first_product_in_runs(gpu, kernel, seq, dim, vocab):
     """The same sums in channel-first logits (MatMulVocabSeq), by blocks as above."""
     p = plan.plans([(seq, vocab, dim, 0)])[0]
