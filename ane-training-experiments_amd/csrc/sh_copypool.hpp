@@ -83,7 +83,7 @@ class CopyPool {
     }
 
   private:
-    static constexpr size_t kPart = 128u << 10;   // about 8 us of copying
+    static constexpr size_t kPart = 32u << 10;   // about 2 us of copying, eight in the ring's least chunk
     static constexpr size_t kMaxParts = 64;
     static constexpr std::chrono::microseconds kSpin{50};   // about the time PCIe takes for a 2 MiB chunk
 

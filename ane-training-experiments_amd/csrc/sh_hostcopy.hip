@@ -17,11 +17,12 @@
 namespace sh {
 namespace {
 
-// Smaller copies take the runtime's own path. Into warm pages, called every 2 ms (the helpers asleep):
-// 1 MiB 63 us by the runtime and 80 through the ring, 2 MiB 122 and 129, 3 MiB 185 and 131, 32 MiB
-// 1878 and 707; into fresh pages 2 MiB 480 and 362. (The other way the runtime is as fast up to 16
-// MiB: 2 MiB in 80 us against 201 through the ring.)
-constexpr size_t kMin = 2u << 20;
+// Smaller copies take the runtime's own path: 0.25 MiB alone 22 us against 47 through the ring with the
+// helpers asleep. Whole calls, three models in turn, by the runtime and through the ring: a layer over
+// 180 rows (0.55 MB) 167 us and 139, over 640 (2 MB) 350 and 287; logits of 5 rows (0.64 MB) 231 us
+// and 226, of 20 (2.6 MB) 346 and 284. (The other way the runtime is as fast up to 16 MiB: 2 MiB in 80
+// us against 201 through the ring.)
+constexpr size_t kMin = 512u << 10;
 // The ring and the threads are set up once a process has copied this much without them: it takes 0.5
 // to 2 ms, mostly of pinning, against about 1 ms that they save per 32 MiB.
 constexpr size_t kSetUp = 32u << 20;

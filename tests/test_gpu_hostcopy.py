@@ -1,5 +1,5 @@
 """Large results copied to host arrays (HostCopier) bit for bit: sizes around its threshold
-(2 MiB), of an uneven last chunk and beyond its pinned ring (8 MiB), at unaligned host
+(512 KiB), of an uneven last chunk and beyond its pinned ring (8 MiB), at unaligned host
 addresses, through a trainer's embedding [V, D] read back. The ring and its threads come with the
 copies that need them, not with a model, are one for all models, and go with the last that used
 them; models on two threads return what each returns alone."""
@@ -16,7 +16,7 @@ from helpers import tiny_config
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("vocab", [2048, 8188, 8192, 8196, 9004, 32772, 65532])   # rows of 256 bytes
+@pytest.mark.parametrize("vocab", [1024, 2044, 2048, 2052, 8188, 9004, 32772, 65532])   # rows of 256 bytes
 def test_read_round_trip(gpu, vocab):
     cfg = tiny_config(dim=64, hidden=128, n_layers=1, n_heads=4, n_kv_heads=4, head_dim=16, vocab=vocab, max_seq=32)
     tr = sh.Trainer(cfg, seq=16)
@@ -52,7 +52,7 @@ def test_threads_come_with_large_copies(gpu):
     before = threads()
     a, _ = wide_model()
     a.greedy_decode(toks[:9], 4)
-    a.eval_logits(toks[:32])          # 1 MiB
+    a.eval_logits(toks[:15])          # 480 KiB
     assert threads() == before
     b, _ = wide_model()
     for m in (a, b):
